@@ -556,6 +556,21 @@ int upload_plan(hmvm_plan* p) {
     UP(ql, L.ql);
     UP(ql_il, L.ql_il);
 #undef UP
+    D.zrel = D.qrel = D.zscale;
+    D.vrel = D.vscale;
+    D.trel = D.tmul;
+    if (!L.rows64 && !L.qmax.empty()) {
+        RelScales S;
+        relative_scales(L, S);
+        if ((rc = upload(p, S.zrel, &D.zrel)) != HMVM_OK) return rc;
+        D.qrel = D.zrel;
+        if (!S.qrel.empty()) {
+            if ((rc = upload(p, S.qrel, &D.qrel)) != HMVM_OK) return rc;
+            if ((rc = upload(p, L.qmax, &D.qmax)) != HMVM_OK) return rc;
+        }
+        if ((rc = upload(p, S.vrel, &D.vrel)) != HMVM_OK) return rc;
+        if ((rc = upload(p, S.trel, &D.trel)) != HMVM_OK) return rc;
+    }
     D.npl = int64_t(L.pl.size());
     D.nql = int64_t(L.ql.size());
     std::vector<RtItem> items;
@@ -592,7 +607,7 @@ int upload_plan(hmvm_plan* p) {
     D.ncols = L.ncols;
     // a workgroup per pack while a wave per pack leaves wave slots idle (4 per
     // SIMD); FP64 only: the FP32 sums keep their order of addition
-    D.rsplit = (D.nrp <= kWidePanels && (L.only_f64() || L.nvals[F64] == 0)) ? 1 : 0;
+    D.rsplit = (D.nrp <= kWidePanels && (L.only_f64() || !L.rows64)) ? 1 : 0;
     D.vsplit = (L.only_f64() && D.nvpacks <= kSplitPacks) ? 1 : 0;
     // the host copies of the arenas are no longer needed on the device path
     L.release_arenas();
@@ -699,7 +714,7 @@ inline int mm_family(const HostLayout& L) { return L.only_f64() ? int(kFamF64) :
 // layout, so that host-only plans answer too)
 int64_t mm_ws_doubles(const hmvm_plan* p, bool trans, int R) {
     const HostLayout& L = p->L;
-    return mrhs_ws_doubles(mm_family(L), L.nvals[F64] > 0, trans ? L.qsize : L.psize, L.ntent,
+    return mrhs_ws_doubles(mm_family(L), L.rows64, trans ? L.qsize : L.psize, L.ntent,
                            trans ? L.nrows : L.ncols, R);
 }
 
@@ -747,14 +762,13 @@ int apply_impl(const hmvm_plan* p, double alpha, int op, const void* x, int64_t 
     int pass = mm_pass(p, trans, nrhs);
     while (pass > 1 && mm_ws_doubles(p, trans, pass) > ws_bytes / int64_t(sizeof(double))) --pass;
     const int fam = mm_family(p->L);
-    const bool has64 = p->L.nvals[F64] > 0;
     for (int r0 = 0; r0 < nrhs; r0 += pass) {
         const int R = std::min(pass, nrhs - r0);
         const void* xr = static_cast<const char*>(x) + size_t(r0) * size_t(ldx) * es;
         void* yr = static_cast<char*>(y) + size_t(r0) * size_t(ldy) * es;
         int rc;
         if (R > 1)
-            rc = launch_apply_mrhs(p->dp, fam, has64, trans, alpha, xr, ldx, yr, ldy, R, vdt, static_cast<double*>(ws),
+            rc = launch_apply_mrhs(p->dp, fam, p->L.rows64, trans, alpha, xr, ldx, yr, ldy, R, vdt, static_cast<double*>(ws),
                                    st) == 0 ? HMVM_OK : HMVM_ERR_DEVICE;
         else if (vdt == HMVM_F64)
             rc = launch_apply(p, alpha, op, static_cast<const double*>(xr), static_cast<double*>(yr),

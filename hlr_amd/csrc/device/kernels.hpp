@@ -30,6 +30,14 @@ struct DevPlan {
     const int32_t* vsrc;
     const float* vscale;      // null: all 1
     const double* tmul;
+    // scale tables of products with several right-hand sides: those above, or
+    // quotients by each entry's (qmax: dense column's) largest scale where the
+    // workspace rows are FP32 (RelScales)
+    const float* zrel;
+    const float* qrel;        // transposed R pass
+    const float* vrel;
+    const float* qmax;        // null: all 1
+    const double* trel;
     const int32_t* pt_off;
     const int32_t* pt_cnt;
     const int32_t* qt_off;

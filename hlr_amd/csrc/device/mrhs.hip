@@ -62,7 +62,7 @@ __global__ __launch_bounds__(256) void k_psum_mm(DevPlan D, const int32_t* __res
                                                  WT* __restrict__ t, int Rs) {
     constexpr int NP = 16 / int(sizeof(WT));
     const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    psum_mm_items<NP, WT, 1, kPsumRound>(D, off, cnt, Pb, t, Rs, 1.0, g, 0, D.ntent * (Rs / NP));
+    psum_mm_items<NP, WT, 1, kPsumRound>(D, D.trel, off, cnt, Pb, t, Rs, 1.0, g, 0, D.ntent * (Rs / NP));
 }
 
 template <int NW, int NTM, typename YT, typename KIND, typename WT = typename KIND::WT>
@@ -92,7 +92,7 @@ inline int64_t pad32(int64_t v) { return (v + 31) / 32 * 32; }
 
 } // namespace
 
-int launch_apply_mrhs(const DevPlan& D, int fam, bool has64, bool trans, double alpha, const void* x, int64_t ldx,
+int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double alpha, const void* x, int64_t ldx,
                       void* y, int64_t ldy, int R, int vdt, double* ws, hipStream_t st) {
     if (R < 2 || R > kMaxRp) return 1;
     if (fam != kFamHw && fam != kFamBfp && fam != kFamF64 && fam != kFamAfl) return 1;
@@ -141,7 +141,7 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool has64, bool trans, double 
     // accumulators sized for exactly the ceil(R / 16) tiles of this call; one
     // instantiation per kind of plan, which carries only its own formats'
     // decode paths (and registers)
-    by_mm_kind(fam, has64, [&](auto kind) {
+    by_mm_kind(fam, rows64, [&](auto kind) {
         auto with = [&](auto ntm) {
             if (vdt == 0) run(kind, ntm, double(0));
             else run(kind, ntm, float(0));
@@ -156,8 +156,8 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool has64, bool trans, double 
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-int64_t mrhs_ws_doubles(int fam, bool has64, int64_t partials, int64_t ntent, int64_t nin, int R) {
-    const bool f = mm_float_rows(fam, has64);
+int64_t mrhs_ws_doubles(int fam, bool rows64, int64_t partials, int64_t ntent, int64_t nin, int R) {
+    const bool f = mm_float_rows(fam, rows64);
     const int64_t Rs = f ? rhs_stride<float>(R) : rhs_stride<double>(R);
     const int64_t rows = ntent + nin + 1;
     // z rows are addressed with 32-bit byte offsets

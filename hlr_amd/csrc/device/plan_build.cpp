@@ -267,6 +267,65 @@ float fp8_scale(double maxabs) {
     return s;
 }
 
+bool all_zero(const double* v, int64_t m) {
+    for (int64_t i = 0; i < m; ++i)
+        if (v[i] != 0) return false;
+    return true;
+}
+
+// The largest scales per t-entry and global column, and whether workspace
+// rows in FP32 keep the range that the products of one right-hand side have.
+// FP32 rows hold values relative to these (P / vmax, Q / zmax or qmax, t vmax
+// zmax): they are then FP32 sums themselves or what FP32 arithmetic takes
+// them to, so nothing leaves FP32's range that did not before.  Two cases
+// keep FP64 rows: scales of one entry more than 2^64 apart, whose quotients
+// would bring small sums near FP32's smallest values, and dense columns of a
+// scaled format at indices that no low-rank leaf covers, whose x is scaled
+// before it is rounded (a low-rank leaf rounds it unscaled).
+void range_scales(HostLayout& L) {
+    L.rows64 = L.nvals[F64] > 0;
+    bool any = false;
+    for (int f = 0; f < NFMT; ++f) any = any || (fmt_scaled(f) && !fmt_is_afl(f) && L.nvals[f] > 0);
+    if (!any || L.rows64) return;
+    L.zmax.assign(size_t(L.ntent), 0.0f);
+    L.vmax.assign(size_t(L.ntent), 0.0f);
+    L.qmax.assign(size_t(L.ncols), 0.0f);
+    std::vector<int32_t> cover(size_t(L.ncols) + 1, 0);
+    for (const hmvm_block& b : L.blocks)
+        if (b.kind != HMVM_BLOCK_DENSE && b.rank > 0) {
+            ++cover[size_t(b.col_ofs)];
+            --cover[size_t(b.col_ofs + b.ncols)];
+        }
+    for (int64_t j = 0; j < L.ncols; ++j) cover[size_t(j) + 1] += cover[size_t(j)];
+    bool bare = false;
+    // calls f(column's maximum, scale) for the nonzero columns
+    auto each = [&](auto&& f) {
+        for (const RChunk& C : L.rchunks) {
+            if (!fmt_scaled(C.fmt)) continue;
+            for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c) {
+                const int32_t s = L.colsrc[size_t(c)];
+                if (s == kPadCol || L.znull[size_t(c)]) continue;
+                bare = bare || (s >= 0 && cover[size_t(s)] == 0);
+                f(s >= 0 ? L.qmax[size_t(s)] : L.zmax[size_t(~s)], L.zscale[size_t(c)]);
+            }
+        }
+        for (const VItem& v : L.fitems) {
+            if (!fmt_scaled(v.fmt)) continue;
+            for (int64_t c = v.vc0; c < v.vc0 + int64_t(v.ng) * fmt_width(v.fmt); ++c) {
+                const int32_t e = L.vsrc[size_t(c)];
+                if (e >= 0 && !L.vnull[size_t(c)]) f(L.vmax[size_t(e)], L.vscale[size_t(c)]);
+            }
+        }
+    };
+    each([](float& m, float s) { m = std::max(m, s); });
+    float least = 1.0f;
+    each([&](float& m, float s) { least = std::min(least, s / m); });
+    L.rows64 = bare || least < 0x1p-64f;
+    for (auto* v : {&L.zmax, &L.vmax, &L.qmax})
+        for (float& m : *v)
+            if (m == 0.0f) m = 1.0f;
+}
+
 struct Seg {              // a block's contribution to one panel
     int64_t b;            // block
     int32_t pi;           // panel index inside the block's panel range
@@ -826,6 +885,8 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
     if (need_scale) {
         L.zscale.assign(nrcols, 1.0f);
         L.vscale.assign(nvcols, 1.0f);
+        L.znull.assign(nrcols, 0);
+        L.vnull.assign(nvcols, 0);
     }
 
     // store m values src[0..m) of one panel column in format f at value
@@ -894,7 +955,7 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
                     const float sc = store_col(f, fbase[f], m, W, c, src);
                     const int64_t gc = rcol0[p][f] + c;
                     L.colsrc[gc] = int32_t(b.col_ofs + j);
-                    if (need_scale) L.zscale[gc] = sc;
+                    if (need_scale) { L.zscale[gc] = sc; L.znull[gc] = all_zero(src, m); }
                     L.rdest[gc] = ddest[dstart[s.b] + int64_t(s.pi) * b.ncols + j];
                 }
             } else {
@@ -906,7 +967,7 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
                     const float sc = store_col(f, fbase[f], m, W, c, src);
                     const int64_t gc = rcol0[p][f] + c;
                     L.colsrc[gc] = ~int32_t(e0 + l);
-                    if (need_scale) L.zscale[gc] = sc;
+                    if (need_scale) { L.zscale[gc] = sc; L.znull[gc] = all_zero(src, m); }
                     L.rdest[gc] = L.qt_off[e0 + l] + s.pi * int32_t(b.rank);
                 }
             }
@@ -934,7 +995,7 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
                     const int64_t vc = sg.vc0 + cc;
                     L.vdest[vc] = L.pt_off[e0 + l] + int32_t(u) * int32_t(b.rank);
                     L.vsrc[vc] = int32_t(e0 + l);
-                    if (need_scale) L.vscale[vc] = sc;
+                    if (need_scale) { L.vscale[vc] = sc; L.vnull[vc] = all_zero(src, sg.m); }
                 }
             }
         }
@@ -959,7 +1020,7 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
                 const int64_t vc = sg.vc0 + cc;
                 L.vdest[vc] = L.pt_off[e0 + l] + sgm.pi * int32_t(b.rank);
                 L.vsrc[vc] = int32_t(e0 + l);
-                if (need_scale) L.vscale[vc] = sc;
+                if (need_scale) { L.vscale[vc] = sc; L.vnull[vc] = all_zero(src, m); }
             }
         }
     }
@@ -996,6 +1057,7 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
         if (int(hw) + int(bfp) + int(aflf) > 1) return HMVM_ERR_INVALID_ARG;
         L.family = bfp ? kFamBfp : aflf ? kFamAfl : kFamHw;
     }
+    range_scales(L);
     // bytes per stored value (16 bytes per row of W values)
     auto vbytes = [](int f) { return 16.0 / double(fmt_width(f)); };
     double fl = 0, ds = 0, br = 0, bv = 0;
@@ -1038,6 +1100,40 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
     L.flops = fl;
     L.datasize = ds;
     return HMVM_OK;
+}
+
+// The scale tables of FP32 workspace rows (range_scales): quotients of powers
+// of two.  zrel: R columns, forward (dense columns keep their own scale, which
+// multiplies x); qrel: the same, transposed; vrel: V columns; trel: tmul with
+// the entry's largest scales.
+void relative_scales(const HostLayout& L, RelScales& S) {
+    S.zrel = L.zscale;
+    S.vrel = L.vscale;
+    S.trel = L.tmul;
+    for (int64_t e = 0; e < L.ntent; ++e) S.trel[size_t(e)] *= double(L.zmax[size_t(e)]) * double(L.vmax[size_t(e)]);
+    bool dense = false;
+    for (const RChunk& C : L.rchunks) {
+        if (!fmt_scaled(C.fmt)) continue;
+        for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c) {
+            const int32_t s = L.colsrc[size_t(c)];
+            if (s < 0 && s != kPadCol) S.zrel[size_t(c)] /= L.zmax[size_t(~s)];
+            dense = dense || s >= 0;
+        }
+    }
+    for (const VItem& v : L.fitems) {
+        if (!fmt_scaled(v.fmt)) continue;
+        for (int64_t c = v.vc0; c < v.vc0 + int64_t(v.ng) * fmt_width(v.fmt); ++c) {
+            const int32_t e = L.vsrc[size_t(c)];
+            if (e >= 0) S.vrel[size_t(c)] /= L.vmax[size_t(e)];
+        }
+    }
+    if (!dense) return;
+    S.qrel = S.zrel;
+    for (const RChunk& C : L.rchunks) {
+        if (!fmt_scaled(C.fmt)) continue;
+        for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c)
+            if (L.colsrc[size_t(c)] >= 0) S.qrel[size_t(c)] /= L.qmax[size_t(L.colsrc[size_t(c)])];
+    }
 }
 
 // ---------------------------------------------------------------------------

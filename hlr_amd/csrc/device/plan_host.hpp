@@ -40,6 +40,13 @@ struct HostLayout {
     std::vector<int64_t> blk_d0;   // per block: first dense column in dfmt (-1 for low-rank)
     std::vector<int8_t> dfmt;      // per dense column (block by block): storage format
     std::vector<double> tmul;      // per t-entry: S_l for U S V^T leaves, else 1
+    // largest scale of the nonzero panel columns of t-entry e (R and V side)
+    // and of the dense columns of global column j (empty: no scaled columns)
+    std::vector<float> zmax, vmax, qmax;
+    std::vector<uint8_t> znull, vnull;     // panel columns whose stored values are all zero
+    // Workspace rows of several right-hand sides in FP64: FP64 values are
+    // stored, or FP32 rows would narrow the range of the vectors (range_scales)
+    bool rows64 = false;
     std::vector<int32_t> pt_off, pt_cnt;   // forward partials of t-entry e
     std::vector<int32_t> qt_off, qt_cnt;   // transposed partials of t-entry e
     std::vector<int32_t> tstride;          // distance of consecutive partials of e (= rank)
@@ -93,6 +100,8 @@ struct HostLayout {
         std::vector<uint16_t>().swap(a16);
         std::vector<uint8_t>().swap(a8);
         for (auto& v : abfp) std::vector<uint32_t>().swap(v);
+        for (auto* v : {&zmax, &vmax, &qmax}) std::vector<float>().swap(*v);
+        for (auto* v : {&znull, &vnull}) std::vector<uint8_t>().swap(*v);
     }
 };
 
@@ -100,6 +109,13 @@ struct HostLayout {
 int build_layout(const hmvm_block* blocks, int64_t nblocks, int64_t nrows, int64_t ncols,
                  const double* arena, int64_t arena_len, const hmvm_plan_opts& opts,
                  HostLayout& L);
+
+// scale tables of FP32 workspace rows, for plans with zmax, vmax, qmax
+struct RelScales {
+    std::vector<float> zrel, vrel, qrel;   // qrel empty: zrel (no scaled dense columns)
+    std::vector<double> trel;
+};
+void relative_scales(const HostLayout& L, RelScales& S);
 
 // dequantise one block's factors from (host copies of) the arenas
 int unpack_block(const HostLayout& L, int64_t b, const void* const arenas[NFMT], bool as_f64, double* a, double* bb);
