@@ -714,15 +714,29 @@ inline int mm_family(const HostLayout& L) { return L.only_f64() ? int(kFamF64) :
 // layout, so that host-only plans answer too)
 int64_t mm_ws_doubles(const hmvm_plan* p, bool trans, int R) {
     const HostLayout& L = p->L;
-    return mrhs_ws_doubles(mm_family(L), L.rows64, trans ? L.qsize : L.psize, L.ntent,
+    return mrhs_ws_doubles(mm_family(L), L.rows64, trans, trans ? L.qsize : L.psize, L.ntent,
                            trans ? L.nrows : L.ncols, R);
 }
 
-// right-hand sides per pass of a call: at most kMrhsMax, and what the
-// kernels' offsets reach
-int mm_pass(const hmvm_plan* p, bool trans, int nrhs) {
-    int pass = std::min(nrhs, kMrhsMax);
-    while (pass > 1 && mm_ws_doubles(p, trans, pass) == INT64_MAX) --pass;
+constexpr int64_t kNoallocDoubles = HMVM_NOALLOC_MAX_BYTES / int64_t(sizeof(double));
+
+// right-hand sides of a group of G (2 .. kMrhsMax) that one pass on the matrix
+// cores takes: as many as `room` doubles of workspace and the kernels' offsets
+// hold; 0: the group runs one vector at a time.
+//
+// A column's result does not depend on the others of its pass, so that any
+// split gives the same bits, and a call with a small workspace
+// (hmvm_apply_noalloc) those of hmvm_apply.  Hence a pass may have one column,
+// and the columns that take the single-vector kernels are chosen by the number
+// of right-hand sides alone: those of a group of one.  The second condition
+// keeps this for plans with fewer t entries than rows whose transposed product
+// fits the fixed array with the single-vector kernels only.
+int mm_pass(const hmvm_plan* p, bool trans, int G, int64_t room) {
+    if (G < 2) return 0;
+    if (trans && ws_doubles(p, HMVM_OP_TRANSPOSED) <= kNoallocDoubles && mm_ws_doubles(p, trans, 1) > kNoallocDoubles)
+        return 0;
+    int pass = G;
+    while (pass > 0 && mm_ws_doubles(p, trans, pass) > room) --pass;
     return pass;
 }
 
@@ -745,8 +759,8 @@ int64_t min_ws_doubles(const hmvm_plan* p, int op, int nrhs) {
 int64_t call_ws_doubles(const hmvm_plan* p, int op, int nrhs) {
     const bool trans = (op == HMVM_OP_TRANSPOSED || op == HMVM_OP_ADJOINT);
     const int64_t w = min_ws_doubles(p, op, nrhs);
-    const int pass = mm_pass(p, trans, nrhs);
-    return pass > 1 ? std::max(w, mm_ws_doubles(p, trans, pass)) : w;
+    const int pass = mm_pass(p, trans, std::min(nrhs, kMrhsMax), INT64_MAX - 1);
+    return pass > 0 ? std::max(w, mm_ws_doubles(p, trans, pass)) : w;
 }
 
 int apply_impl(const hmvm_plan* p, double alpha, int op, const void* x, int64_t ldx, void* y, int64_t ldy,
@@ -757,26 +771,29 @@ int apply_impl(const hmvm_plan* p, double alpha, int op, const void* x, int64_t 
     if (nrhs > 1 && (ldx < nin || ldy < nout)) return HMVM_ERR_LAYOUT;
     if (ws_bytes < min_ws_doubles(p, op, nrhs) * int64_t(sizeof(double))) return HMVM_ERR_INVALID_ARG;
     const size_t es = (vdt == HMVM_F64) ? 8 : 4;
-    // matrix cores, up to kMrhsMax right-hand sides per pass, as many as the
-    // workspace holds; one vector at a time where that is one
-    int pass = mm_pass(p, trans, nrhs);
-    while (pass > 1 && mm_ws_doubles(p, trans, pass) > ws_bytes / int64_t(sizeof(double))) --pass;
     const int fam = mm_family(p->L);
-    for (int r0 = 0; r0 < nrhs; r0 += pass) {
-        const int R = std::min(pass, nrhs - r0);
+    auto part = [&](int r0, int R, bool mm) -> int {
         const void* xr = static_cast<const char*>(x) + size_t(r0) * size_t(ldx) * es;
         void* yr = static_cast<char*>(y) + size_t(r0) * size_t(ldy) * es;
-        int rc;
-        if (R > 1)
-            rc = launch_apply_mrhs(p->dp, fam, p->L.rows64, trans, alpha, xr, ldx, yr, ldy, R, vdt, static_cast<double*>(ws),
-                                   st) == 0 ? HMVM_OK : HMVM_ERR_DEVICE;
-        else if (vdt == HMVM_F64)
-            rc = launch_apply(p, alpha, op, static_cast<const double*>(xr), static_cast<double*>(yr),
-                              static_cast<double*>(ws), st);
-        else
-            rc = launch_apply(p, alpha, op, static_cast<const float*>(xr), static_cast<float*>(yr),
-                              static_cast<double*>(ws), st);
-        if (rc != HMVM_OK) return rc;
+        if (mm)
+            return launch_apply_mrhs(p->dp, fam, p->L.rows64, trans, alpha, xr, ldx, yr, ldy, R, vdt,
+                                     static_cast<double*>(ws), st) == 0 ? HMVM_OK : HMVM_ERR_DEVICE;
+        if (vdt == HMVM_F64)
+            return launch_apply(p, alpha, op, static_cast<const double*>(xr), static_cast<double*>(yr),
+                                static_cast<double*>(ws), st);
+        return launch_apply(p, alpha, op, static_cast<const float*>(xr), static_cast<float*>(yr),
+                            static_cast<double*>(ws), st);
+    };
+    // groups of up to kMrhsMax right-hand sides, each in equal parts that the
+    // workspace holds
+    for (int g0 = 0; g0 < nrhs; g0 += kMrhsMax) {
+        const int G = std::min(kMrhsMax, nrhs - g0);
+        const int pass = mm_pass(p, trans, G, ws_bytes / int64_t(sizeof(double)));
+        const int parts = pass > 0 ? (G + pass - 1) / pass : G, per = (G + parts - 1) / parts;
+        for (int r0 = 0; r0 < G; r0 += per) {
+            const int rc = part(g0 + r0, std::min(per, G - r0), pass > 0);
+            if (rc != HMVM_OK) return rc;
+        }
     }
     return HMVM_OK;
 }
@@ -1029,13 +1046,12 @@ int hmvm_apply(const hmvm_plan* p, double alpha, int op, const void* x, int64_t 
     hipStream_t st = static_cast<hipStream_t>(stream);
     int64_t bytes = call_ws_doubles(p, op, nrhs) * int64_t(sizeof(double));
     void* ws = nullptr;
-    if (hipMallocAsync(&ws, size_t(bytes), st) != hipSuccess) {
-        // no room for all right-hand sides of a pass at once
-        const int64_t least = min_ws_doubles(p, op, nrhs) * int64_t(sizeof(double));
-        if (least >= bytes) return HMVM_ERR_ALLOC;
+    // no room for all right-hand sides of a pass at once: fewer
+    const int64_t least = min_ws_doubles(p, op, nrhs) * int64_t(sizeof(double));
+    while (hipMallocAsync(&ws, size_t(bytes), st) != hipSuccess) {
+        if (bytes <= least) return HMVM_ERR_ALLOC;
         (void)hipGetLastError();
-        bytes = least;
-        if (hipMallocAsync(&ws, size_t(bytes), st) != hipSuccess) return HMVM_ERR_ALLOC;
+        bytes = std::max(least, bytes / 2);
     }
     rc = apply_impl(p, alpha, op, x, ldx, y, ldy, nrhs, vdt, ws, bytes, st);
     if (hipFreeAsync(ws, st) != hipSuccess && rc == HMVM_OK) rc = HMVM_ERR_DEVICE;

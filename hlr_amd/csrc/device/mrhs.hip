@@ -19,6 +19,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <type_traits>
 
@@ -55,12 +56,12 @@ __global__ __launch_bounds__(kThr, (mm_rtrn_waves<NTM, KIND>())) void k_rtrn_mm(
     rchunk_trn_mm<NTM, KIND::FAM, WT>(P, C, XTb, Rs, Q, tiles[wave], wave, threadIdx.x & 63);
 }
 
-// one item (entry, 16-byte unit of right-hand sides) per thread
-template <typename WT>
+// one item (entry, NP right-hand sides: a 16-byte unit, or the only one) per
+// thread
+template <int NP, typename WT>
 __global__ __launch_bounds__(256) void k_psum_mm(DevPlan D, const int32_t* __restrict__ off,
                                                  const int32_t* __restrict__ cnt, const WT* __restrict__ Pb,
                                                  WT* __restrict__ t, int Rs) {
-    constexpr int NP = 16 / int(sizeof(WT));
     const int64_t g = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     psum_mm_items<NP, WT, 1, kPsumRound>(D, D.trel, off, cnt, Pb, t, Rs, 1.0, g, 0, D.ntent * (Rs / NP));
 }
@@ -88,13 +89,11 @@ __global__ __launch_bounds__(kThr, (mm_vtrn_waves<NTM, KIND>())) void k_vtrn_mm(
                                           threadIdx.x & 63);
 }
 
-inline int64_t pad32(int64_t v) { return (v + 31) / 32 * 32; }
-
 } // namespace
 
 int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double alpha, const void* x, int64_t ldx,
                       void* y, int64_t ldy, int R, int vdt, double* ws, hipStream_t st) {
-    if (R < 2 || R > kMaxRp) return 1;
+    if (R < 1 || R > kMaxRp) return 1;
     if (fam != kFamHw && fam != kFamBfp && fam != kFamF64 && fam != kFamAfl) return 1;
     const int64_t nin = trans ? D.nrows : D.ncols;
     auto blocks = [](int64_t n, int per) { return unsigned((n + per - 1) / per); };
@@ -105,10 +104,13 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double
         constexpr int NTM = decltype(ntm)::value;
         constexpr int NP = 16 / int(sizeof(WT));
         const int Rs = rhs_stride<WT>(R);
-        // workspace, rows of Rs values at 16-byte boundaries: partials | t | XT
+        // workspace, rows of Rs values at 16-byte boundaries: partials | z rows.
+        // Forward: t | XT (zero row last).  Transposed: t takes the place of
+        // XT, which the sums no longer need; XT lies at its end, so that the
+        // zero row stays behind both.
         WT* part = reinterpret_cast<WT*>((reinterpret_cast<uintptr_t>(ws) + 15) & ~uintptr_t(15));
         WT* t = part + (trans ? D.qsize : D.psize) * Rs;
-        WT* xt = t + D.ntent * Rs;
+        WT* xt = t + (trans ? trn_zero_row(D) - nin : D.ntent) * Rs;
         YT* Y = static_cast<YT*>(y);
         k_xtrans<YT, WT><<<unsigned(xtrans_tiles(nin)), kThr, xtrans_lds_bytes(R), st>>>(static_cast<const YT*>(x), ldx,
                                                                                          nin, R, xt);
@@ -117,9 +119,14 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double
         } else {
             if (D.nfitems > 0) k_vfwd_mm<NTM, KIND><<<unsigned(D.nfitems), kThr, 0, st>>>(D, xt, Rs, part);
         }
-        if (D.ntent > 0)
-            k_psum_mm<WT><<<blocks(D.ntent * (Rs / NP), 256), 256, 0, st>>>(D, trans ? D.qt_off : D.pt_off,
-                                                                            trans ? D.qt_cnt : D.pt_cnt, part, t, Rs);
+        if (D.ntent > 0) {
+            const int32_t* off = trans ? D.qt_off : D.pt_off;
+            const int32_t* cnt = trans ? D.qt_cnt : D.pt_cnt;
+            if (R > 1)
+                k_psum_mm<NP, WT><<<blocks(D.ntent * (Rs / NP), 256), 256, 0, st>>>(D, off, cnt, part, t, Rs);
+            else
+                k_psum_mm<1, WT><<<blocks(D.ntent, 256), 256, 0, st>>>(D, off, cnt, part, t, Rs);
+        }
         if (trans) {
             if (D.ncp > 0)
                 k_vtrn_mm<NTM, YT, KIND><<<unsigned(D.ncp), kThr, mm_red_bytes(kThr / 64), st>>>(D, alpha, t, part, Y, ldy, R);
@@ -156,10 +163,10 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double
     return hipGetLastError() == hipSuccess ? 0 : 2;
 }
 
-int64_t mrhs_ws_doubles(int fam, bool rows64, int64_t partials, int64_t ntent, int64_t nin, int R) {
+int64_t mrhs_ws_doubles(int fam, bool rows64, bool trans, int64_t partials, int64_t ntent, int64_t nin, int R) {
     const bool f = mm_float_rows(fam, rows64);
     const int64_t Rs = f ? rhs_stride<float>(R) : rhs_stride<double>(R);
-    const int64_t rows = ntent + nin + 1;
+    const int64_t rows = (trans ? std::max(ntent, nin) : ntent + nin) + 1;
     // z rows are addressed with 32-bit byte offsets
     if (rows * Rs * (f ? 4 : 8) > int64_t(UINT32_MAX)) return INT64_MAX;
     return (partials + rows) * Rs / (f ? 2 : 1) + 2;

@@ -213,9 +213,13 @@ int hmvm_apply_timed(const hmvm_plan* plan, double alpha, int op,
                      float ms[3]);
 
 /* bytes of workspace of a call (op, nrhs): with this much, hmvm_apply_ws takes
- * up to 64 right-hand sides per pass over the factors.  A transposed call with
- * nrhs > 1 also accepts less, down to the size for nrhs = 1, and then takes
- * fewer right-hand sides per pass. */
+ * up to 64 right-hand sides per pass over the factors.  A call with nrhs > 1
+ * also accepts less and then takes fewer right-hand sides per pass: down to the
+ * size for nrhs = 1 (transposed), or to that of min(nrhs, 64) right-hand sides
+ * in rows without padding (forward).  The number per pass does not change the
+ * results of a column, unless a transposed call has less than one column
+ * takes on the matrix cores: its vectors then run one at a time and the
+ * results agree up to rounding. */
 int hmvm_workspace_size(const hmvm_plan* plan, int op, int nrhs, int64_t* bytes);
 
 /* hmvm_apply with a caller-provided device workspace (no allocation) */
@@ -233,12 +237,12 @@ int hmvm_apply_ws(const hmvm_plan* plan, double alpha, int op,
  * HMVM_NOALLOC_MAX_BYTES that the library holds on every GPU it runs on
  * until the process ends.  Arguments and results are those of hmvm_apply,
  * with the same kernels, so the results are bitwise those of hmvm_apply.
- * A call whose smallest workspace exceeds HMVM_NOALLOC_MAX_BYTES fails with
- * HMVM_ERR_TOO_LARGE before any device work; a transposed call whose
- * hmvm_workspace_size exceeds it takes fewer right-hand sides per pass (one at
- * a time, equal to hmvm_apply up to rounding, where two do not fit).  All calls on one GPU share that GPU's array: calls that overlap in
- * time on one GPU (different streams or host threads) race and give wrong
- * results; serialise them.  No counterpart in the reference: it is for
+ * A call whose smallest workspace (see hmvm_workspace_size) exceeds
+ * HMVM_NOALLOC_MAX_BYTES fails with HMVM_ERR_TOO_LARGE before any device work;
+ * one whose full workspace exceeds it takes fewer right-hand sides per pass
+ * over the factors, with the same bits.  All calls on one GPU share that GPU's
+ * array: calls that overlap in time on one GPU (different streams or host
+ * threads) race and give wrong results; serialise them.  No counterpart in the reference: it is for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid allocation).
  */
