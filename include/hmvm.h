@@ -331,13 +331,14 @@ int hmvm_batch_destroy(hmvm_batch* batch);
 /*
  * y_i += alpha_i A_i x_i for every plan i (forward products; nrhs[i] in
  * 1..64 right-hand sides, column-major with ldx[i] / ldy[i]).  The work of
- * all members runs as a fixed sequence of at most sixteen stream-ordered
- * kernels (transposed copy of X, column-panel pass for one and for several
- * right-hand sides, two partial-sum stages, row-panel pass for one and for
- * several right-hand sides; the matrix-core passes once per count of
- * 16-wide right-hand-side tiles), one unit of work per workgroup, whatever
- * the number of members.  No counterpart in the
- * reference (it applies one matrix at a time, programs/mvm/mvm.hh:151-204).
+ * all members runs as stream-ordered kernels, one unit of work per workgroup:
+ * transposed copy of X, column-panel passes, partial sums, row-panel passes,
+ * one kernel per count of 16-wide right-hand-side tiles and waves per panel: at
+ * most sixteen kernels whatever the number of members.  Every member runs the
+ * arithmetic of its own plan, whatever the others are stored in: with several
+ * right-hand sides its result has the bits of hmvm_apply.
+ * No counterpart in the reference (it applies one matrix at a time,
+ * programs/mvm/mvm.hh:151-204).
  */
 int hmvm_batch_apply(hmvm_batch* batch, const double* alphas,
                      const void* const* xs, const int64_t* ldx,
