@@ -337,6 +337,10 @@ int hmvm_batch_destroy(hmvm_batch* batch);
  * most sixteen kernels whatever the number of members.  Every member runs the
  * arithmetic of its own plan, whatever the others are stored in: with several
  * right-hand sides its result has the bits of hmvm_apply.
+ * The y of two members must not overlap, nor a y and the x of another member,
+ * unless one of them has one right-hand side and the other several, or their
+ * counts of 16-wide tiles differ: members then act on y in the order of these
+ * counts, those of one right-hand side first.
  * No counterpart in the reference (it applies one matrix at a time,
  * programs/mvm/mvm.hh:151-204).
  */
