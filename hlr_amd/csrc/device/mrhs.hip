@@ -4,15 +4,16 @@
 // single right-hand-side path, with the inner products done as 16 x 16 x 4
 // MFMA tiles:
 //   forward     V pass -> partial sums -> R pass
+//   transposed  R pass -> partial sums -> V pass
 //               FP64 factors v_mfma_f64_16x16x4f64, the other formats
-//               decoded to FP32, v_mfma_f32_16x16x4f32
-//   transposed  R pass -> partial sums -> V pass, FP64 tiles for every format
+//               decoded to FP32, v_mfma_f32_16x16x4f32; the transposed V pass
+//               FP64 tiles for every format
 // Right-hand sides are processed in tiles of 16.
 //
 //   k_xtrans   XT = X^T, the right-hand sides of an index contiguous
 //   k_vfwd_mm  P(c, r) = sum_i V(i, c) X(i, r)      workgroup per V segment
 //   k_rtrn_mm  Q(c, r) = sum_i R(i, c) X(i, r)      workgroup per R chunk
-//   k_psum_mm  t_e = S_e sum of the entry's partials
+//   k_psum_mm  t_e = S_e sum of the entry's partials (FP64 sums)
 //   k_ufwd_mm  Y(i, r) += a sum_c R(i, c) Z(c, r)   workgroup per row panel
 //   k_vtrn_mm  Y(i, r) += a (sum_c V(i, c) t_c + dense partials)
 //                                                   workgroup per column panel
