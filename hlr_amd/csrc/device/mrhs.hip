@@ -57,8 +57,7 @@ __global__ __launch_bounds__(kThr, (mm_rtrn_waves<NTM, KIND>())) void k_rtrn_mm(
     rchunk_trn_mm<NTM, KIND::FAM, WT>(P, C, XTb, Rs, Q, tiles[wave], wave, threadIdx.x & 63);
 }
 
-// one item (entry, NP right-hand sides: a 16-byte unit, or the only one) per
-// thread
+// one item (entry, NP right-hand sides: a unit of rhs_unit) per thread
 template <int NP, typename WT>
 __global__ __launch_bounds__(256) void k_psum_mm(DevPlan D, const int32_t* __restrict__ off,
                                                  const int32_t* __restrict__ cnt, const WT* __restrict__ Pb,
@@ -103,7 +102,6 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double
         using WT = typename KIND::WT;
         using YT = decltype(ytag);
         constexpr int NTM = decltype(ntm)::value;
-        constexpr int NP = 16 / int(sizeof(WT));
         const int Rs = rhs_stride<WT>(R);
         // workspace, rows of Rs values at 16-byte boundaries: partials | z rows.
         // Forward: t | XT (zero row last).  Transposed: t takes the place of
@@ -123,10 +121,15 @@ int launch_apply_mrhs(const DevPlan& D, int fam, bool rows64, bool trans, double
         if (D.ntent > 0) {
             const int32_t* off = trans ? D.qt_off : D.pt_off;
             const int32_t* cnt = trans ? D.qt_cnt : D.pt_cnt;
-            if (R > 1)
+            auto sums = [&](auto np) {
+                constexpr int NP = decltype(np)::value;
                 k_psum_mm<NP, WT><<<blocks(D.ntent * (Rs / NP), 256), 256, 0, st>>>(D, off, cnt, part, t, Rs);
-            else
-                k_psum_mm<1, WT><<<blocks(D.ntent, 256), 256, 0, st>>>(D, off, cnt, part, t, Rs);
+            };
+            switch (rhs_unit<WT>(R)) {
+            case 1: sums(std::integral_constant<int, 1>()); break;
+            case 2: sums(std::integral_constant<int, 2>()); break;
+            default: sums(std::integral_constant<int, 16 / int(sizeof(WT))>()); break;
+            }
         }
         if (trans) {
             if (D.ncp > 0)
