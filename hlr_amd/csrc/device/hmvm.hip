@@ -506,6 +506,11 @@ struct DeviceGuard {
 constexpr size_t kReadPad = 80 * 1024;
 static_assert(kReadPad >= size_t(kPanel) * kItemGroups * 16 + 15 * kPanel * 16, "a tile past the last block");
 
+// at most this many V packs: a workgroup per pack in FP64-only plans, whose
+// single waves stream up to 256 KB each while others of a SIMD have none.  V
+// pass by waves and by workgroups per pack: 293 packs 18.0 / 14.6 us, 1491 30.0
+// / 24.8, 1505 39.4 / 33.9, 3296 53.0 / 47.7, 3433 75.5 / 72.3, 7497 123 / 131.
+// So the line could lie higher, up to about the 4096 waves of four per SIMD.
 constexpr int64_t kSplitPacks = 2048;
 // at most this many row panels: eight waves per panel with several right-hand
 // sides.  Such a plan leaves CUs idle and waits for its longest panel (batch of
@@ -605,9 +610,9 @@ int upload_plan(hmvm_plan* p) {
     D.qsize = L.qsize;
     D.nrows = L.nrows;
     D.ncols = L.ncols;
-    // a workgroup per pack while a wave per pack leaves wave slots idle (4 per
-    // SIMD); FP64 only: the FP32 sums keep their order of addition
+    // the kinds of arithmetic that have the eight-wave form
     D.rsplit = (D.nrp <= kWidePanels && (L.only_f64() || !L.rows64)) ? 1 : 0;
+    // FP64 only: the FP32 sums keep their order of addition
     D.vsplit = (L.only_f64() && D.nvpacks <= kSplitPacks) ? 1 : 0;
     // the host copies of the arenas are no longer needed on the device path
     L.release_arenas();

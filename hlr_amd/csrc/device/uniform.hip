@@ -23,9 +23,8 @@
 // transfers as plain dense leaves in both orientations, so that every step of
 // both products except C^T and N^T is one forward R pass:
 //   A    xc = V^T x (leaf V_c^T), up xc[d-1] += E^T xc[d], C, down, S: y += U yr
-// (n = 32768, 1000 clusters: 170.8 us with 24 launches, 130.7 us).  Large bases
-// (shared bases of big clusters) would leave a few workgroups with whole
-// block rows; their V pass in B splits them by column panels.
+// (n = 32768, 1000 clusters: 170.8 us with 24 launches, 130.7 us), at the price
+// of a second copy of bases and transfers on the device.
 
 #include <hip/hip_runtime.h>
 
@@ -174,7 +173,11 @@ hmvm_block leaf(int64_t r0, int64_t c0, int64_t m, int64_t n, int kind, int64_t 
     return x;
 }
 
-constexpr int64_t kDirectSize = 512;     // rows of the largest explicit basis of a direct plan
+// Rows of the largest explicit basis of a direct plan.  n = 32768, leaf clusters
+// of 64 / 512 / 1024 / 2048: 169 / 328 / 578 / 1253 us with identity leaves, 135
+// / 300 / 558 / 1244 direct.  What is gained is the launches; beyond 512 that is
+// less than 5 % of the product and not worth a second copy of large bases.
+constexpr int64_t kDirectSize = 512;
 
 // the direct plans of one side: analysis, synthesis, upward transfers
 int make_direct(const hmvm_cluster* cb, int64_t n, const Side& s, int64_t dim, const std::vector<double>& ar,

@@ -525,15 +525,17 @@ int hmvm_uplan_create(const hmvm_cluster* rowcb, int64_t nrowcb,
                       const hmvm_plan_opts* opts, int device, hmvm_uplan** out);
 int hmvm_uplan_destroy(hmvm_uplan* plan);
 
-/* statistics: factor bytes of bases, transfers, couplings and dense
-   leaves, mul_vec_flops and mul_vec_datasize (arith/uniform.hh,
-   arith/h2.hh:140-178) */
+/* statistics of the matrix: factor bytes of bases, transfers, couplings and
+   dense leaves, each counted once as FP64, mul_vec_flops and mul_vec_datasize
+   (arith/uniform.hh, arith/h2.hh:140-178).  FP64 plans with explicit bases of at
+   most 512 rows hold bases and transfers in both orientations: their device
+   memory is larger by basis_bytes + transfer_bytes */
 typedef struct hmvm_uplan_info {
     int64_t nrows, ncols;
     int64_t nrow_clusters, ncol_clusters, ncoupling, ndense;
     int32_t nested;              /* 1: H^2 (transfer matrices), 0: uniform-H      */
     int32_t levels;              /* transfer levels (row tree + column tree)      */
-    int64_t basis_bytes;         /* explicit bases, as stored                     */
+    int64_t basis_bytes;         /* explicit bases                                */
     int64_t transfer_bytes;
     int64_t coupling_bytes;
     int64_t dense_bytes;
