@@ -297,30 +297,44 @@ void range_scales(HostLayout& L) {
             --cover[size_t(b.col_ofs + b.ncols)];
         }
     for (int64_t j = 0; j < L.ncols; ++j) cover[size_t(j) + 1] += cover[size_t(j)];
+    // largest and smallest scale of the nonzero columns; each table has one
+    // section that writes it
     bool bare = false;
-    // calls f(column's maximum, scale) for the nonzero columns
-    auto each = [&](auto&& f) {
+    std::vector<float> zmin(L.zmax.size(), FLT_MAX), vmin(L.vmax.size(), FLT_MAX), qmin(L.qmax.size(), FLT_MAX);
+    auto put = [](std::vector<float>& hi, std::vector<float>& lo, size_t k, float s) {
+        hi[k] = std::max(hi[k], s);
+        lo[k] = std::min(lo[k], s);
+    };
+#pragma omp parallel sections
+    {
+#pragma omp section
         for (const RChunk& C : L.rchunks) {
             if (!fmt_scaled(C.fmt)) continue;
             for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c) {
                 const int32_t s = L.colsrc[size_t(c)];
                 if (s == kPadCol || L.znull[size_t(c)]) continue;
                 bare = bare || (s >= 0 && cover[size_t(s)] == 0);
-                f(s >= 0 ? L.qmax[size_t(s)] : L.zmax[size_t(~s)], L.zscale[size_t(c)]);
+                if (s >= 0) put(L.qmax, qmin, size_t(s), L.zscale[size_t(c)]);
+                else put(L.zmax, zmin, size_t(~s), L.zscale[size_t(c)]);
             }
         }
+#pragma omp section
         for (const VItem& v : L.fitems) {
             if (!fmt_scaled(v.fmt)) continue;
             for (int64_t c = v.vc0; c < v.vc0 + int64_t(v.ng) * fmt_width(v.fmt); ++c) {
                 const int32_t e = L.vsrc[size_t(c)];
-                if (e >= 0 && !L.vnull[size_t(c)]) f(L.vmax[size_t(e)], L.vscale[size_t(c)]);
+                if (e >= 0 && !L.vnull[size_t(c)]) put(L.vmax, vmin, size_t(e), L.vscale[size_t(c)]);
             }
         }
+    }
+    bool apart = false;
+    auto far = [&](const std::vector<float>& hi, const std::vector<float>& lo) {
+        for (size_t k = 0; k < hi.size(); ++k) apart = apart || (hi[k] > 0 && lo[k] / hi[k] < 0x1p-64f);
     };
-    each([](float& m, float s) { m = std::max(m, s); });
-    float least = 1.0f;
-    each([&](float& m, float s) { least = std::min(least, s / m); });
-    L.rows64 = bare || least < 0x1p-64f;
+    far(L.zmax, zmin);
+    far(L.vmax, vmin);
+    far(L.qmax, qmin);
+    L.rows64 = bare || apart;
     for (auto* v : {&L.zmax, &L.vmax, &L.qmax})
         for (float& m : *v)
             if (m == 0.0f) m = 1.0f;
@@ -1102,6 +1116,10 @@ int build_layout(const hmvm_block* blocks, int64_t nb, int64_t nrows, int64_t nc
     return HMVM_OK;
 }
 
+// quotient of scales, finite for columns of zeros too, whose scale no maximum
+// counts
+static float quotient(float s, float max) { return std::min(s / max, 0x1p127f); }
+
 // The scale tables of FP32 workspace rows (range_scales): quotients of powers
 // of two.  zrel: R columns, forward (dense columns keep their own scale, which
 // multiplies x); qrel: the same, transposed; vrel: V columns; trel: tmul with
@@ -1111,29 +1129,35 @@ void relative_scales(const HostLayout& L, RelScales& S) {
     S.vrel = L.vscale;
     S.trel = L.tmul;
     for (int64_t e = 0; e < L.ntent; ++e) S.trel[size_t(e)] *= double(L.zmax[size_t(e)]) * double(L.vmax[size_t(e)]);
-    bool dense = false;
-    for (const RChunk& C : L.rchunks) {
-        if (!fmt_scaled(C.fmt)) continue;
-        for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c) {
-            const int32_t s = L.colsrc[size_t(c)];
-            if (s < 0 && s != kPadCol) S.zrel[size_t(c)] /= L.zmax[size_t(~s)];
-            dense = dense || s >= 0;
+    // calls f(R column, its source) for the columns of scaled formats
+    auto each = [&](auto&& f) {
+#pragma omp parallel for schedule(static)
+        for (size_t k = 0; k < L.rchunks.size(); ++k) {
+            const RChunk& C = L.rchunks[k];
+            if (!fmt_scaled(C.fmt)) continue;
+            for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c)
+                if (L.colsrc[size_t(c)] != kPadCol) f(size_t(c), L.colsrc[size_t(c)]);
         }
-    }
-    for (const VItem& v : L.fitems) {
+    };
+    each([&](size_t c, int32_t s) {
+        if (s < 0) S.zrel[c] = quotient(S.zrel[c], L.zmax[size_t(~s)]);
+    });
+#pragma omp parallel for schedule(static)
+    for (size_t k = 0; k < L.fitems.size(); ++k) {
+        const VItem& v = L.fitems[k];
         if (!fmt_scaled(v.fmt)) continue;
         for (int64_t c = v.vc0; c < v.vc0 + int64_t(v.ng) * fmt_width(v.fmt); ++c) {
             const int32_t e = L.vsrc[size_t(c)];
-            if (e >= 0) S.vrel[size_t(c)] /= L.vmax[size_t(e)];
+            if (e >= 0) S.vrel[size_t(c)] = quotient(S.vrel[size_t(c)], L.vmax[size_t(e)]);
         }
     }
+    bool dense = false;
+    for (int8_t f : L.dfmt) dense = dense || fmt_scaled(f);
     if (!dense) return;
     S.qrel = S.zrel;
-    for (const RChunk& C : L.rchunks) {
-        if (!fmt_scaled(C.fmt)) continue;
-        for (int64_t c = C.col0; c < C.col0 + int64_t(C.ngroups) * fmt_width(C.fmt); ++c)
-            if (L.colsrc[size_t(c)] >= 0) S.qrel[size_t(c)] /= L.qmax[size_t(L.colsrc[size_t(c)])];
-    }
+    each([&](size_t c, int32_t s) {
+        if (s >= 0) S.qrel[c] = quotient(S.qrel[c], L.qmax[size_t(s)]);
+    });
 }
 
 // ---------------------------------------------------------------------------

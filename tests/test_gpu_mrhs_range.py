@@ -92,3 +92,30 @@ def test_dense_leaves_in_scaled_formats(cuda, force, op, ed, ex):
         p.apply(1.0, op, X, Y)
         assert np.array_equal(Y.cpu().numpy(), np.broadcast_to(want, Y.shape)), nrhs
     p.close()
+
+
+def test_zero_columns_beside_tiny_ones(cuda):
+    """A column that is zero in one row panel (scale 1) and near the smallest
+    FP8 scales in the other: the quotient of the scales is finite."""
+    import torch
+    m, n, e = 128, 70, -130
+    rng = np.random.default_rng(4)
+    U, V = rng.integers(-4, 5, (m, 2)).astype(np.float64), rng.integers(-4, 5, (n, 2)).astype(np.float64)
+    U[:64, 0] = 0
+    U[64:, 1] = 0
+    b = np.zeros(1, dtype=N.block_dtype())
+    b["nrows"], b["ncols"], b["rank"], b["kind"] = m, n, 2, N.BLOCK_LOWRANK
+    b["off_b"], b["off_s"] = 2 * m, -1
+    arena = np.concatenate([2.0 ** e * U.T.reshape(-1), V.T.reshape(-1)])
+    p = Plan(b, arena, m, n, precision="valr", eps=1e-6, force_format="fp8_e4m3")
+    x = rng.integers(-5, 6, n).astype(np.float64)
+    want = 2.0 ** (e + 60) * (U @ (V.T @ x))
+    for nrhs in (1, 3, 17):
+        print(f"[gpu] mrhs range zero columns nrhs={nrhs}", flush=True)
+        X = torch.as_tensor(np.repeat(2.0 ** 60 * x[None], nrhs, 0), device=cuda)
+        Y = torch.zeros(nrhs, m, dtype=torch.float64, device=cuda)
+        if nrhs == 1:
+            X, Y = X[0], Y[0]
+        p.apply(1.0, N.OP_NORMAL, X, Y)
+        assert np.array_equal(Y.cpu().numpy(), np.broadcast_to(want, Y.shape)), nrhs
+    p.close()
