@@ -5,7 +5,8 @@ plans with per-member numbers of right-hand sides; `apply` runs the work of
 all members as at most sixteen stream-ordered kernels (one unit of work per
 workgroup),
 `capture`/`replay` record that sequence in a HIP graph, `tune` runs the
-in-project autotuner over unit order and partial-sum granularity.
+in-project autotuner over unit order and partial-sum granularity.  The y of
+two members must not overlap (include/hmvm.h has the exceptions).
 """
 from __future__ import annotations
 
